@@ -475,6 +475,12 @@ class Tuner:
         self.cache.put_key(key, res.best, res.best_metric, res.measured)
         return res.best
 
+    def measured_us(self, problem: dict) -> Optional[float]:
+        """The device time of the cached schedule of ``problem``, if it was
+        measured."""
+        e = self.cache.entries.get(problem_key(problem))
+        return e["metric"] * 1e3 if e and e.get("measured") else None
+
     def schedule_for(self, node, mnk) -> MfmaSchedule:
         M, N, K = mnk
         return self.schedule_problem({"kind": "gemm", "M": M, "N": N, "K": K})

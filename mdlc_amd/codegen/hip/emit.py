@@ -39,6 +39,7 @@ epilogue, which also fixes the reference's batch>1 bug (emit.py:187-188).
 
 from __future__ import annotations
 
+from dataclasses import replace
 from typing import Callable, Optional
 
 import numpy as np
@@ -50,7 +51,7 @@ from mdlc_amd.codegen.hip.plan import (LIBRARY_PARTS, QUANT_OPS, HipModule, Laun
 from mdlc_amd.codegen import schedule as schedule_mod
 from mdlc_amd.codegen.schedule import (WINO_BK, WINO_BM, WINO_BN, MfmaSchedule, conv_pool_band,
                                       default_schedule, smallc_fits, smallc_pairs, smallc_tile, split_slices,
-                                      unsplit_if_one_slice, wino_fits,
+                                      unsplit_if_one_slice, wino_fits, x3_schedule, conv_x3_schedule,
                                       wino_patch, wino_pays, wino_slices)
 from mdlc_amd.ir import DType, Graph, Node
 from mdlc_amd.passes.fuse_elementwise import ELEMENTWISE
@@ -64,6 +65,56 @@ REDUCE_VEC = 4        # outputs per thread of the split-K reduce where the layou
 STREAM_K_WGS = 256    # stream-K workgroups: one per CU
 PAIR_MIN_IDLE = 32    # idle CUs a conv's grid must leave for a second conv to share its launch
 SMALLC_WGS = 512      # workgroups stepping through the blocks of the small-channel conv
+
+
+def round8(n: int) -> int:
+    return (int(n) + 7) // 8 * 8
+
+
+def bf16_terms(rem: np.ndarray, img: np.ndarray) -> None:
+    """A contiguous float32 array as three bf16 ones, into img[..., 0 .. 2]
+    (``img`` is the uint16 output with the term axis moved last): each the
+    rounding (nearest, ties to even) of what the ones before leave, so that
+    their sum is the float; infinities and NaNs are the first alone."""
+    finite = bool(np.isfinite(rem).all())
+    for t in range(3):
+        u = rem.view(np.uint32)
+        h = (u >> 16) & 1
+        h += u
+        h += 0x7fff
+        if t == 0:
+            # a finite float whose rounding would overflow is cut instead;
+            # infinities and NaNs stay as they are (a NaN quiet)
+            over = (h & 0x7f800000) == 0x7f800000
+            if not finite or over.any():
+                nan = (u & 0x7fffffff) > 0x7f800000
+                h = np.where(over | nan, u | np.where(nan, np.uint32(0x400000), np.uint32(0)), h)
+        img[..., t] = h >> 16
+        if t < 2:
+            h &= 0xffff0000
+            if t == 0 and not finite:
+                with np.errstate(invalid="ignore"):
+                    rem = np.where(np.isfinite(rem), rem - h.view(np.float32), np.float32(0))
+            else:
+                rem = rem - h.view(np.float32)
+
+
+def x3_pack(mat: np.ndarray) -> tuple:
+    """A float32 matrix [rows][K] as ``gemm_x3`` reads it: (uint16 image
+    [rows / 32][K / 16][h, m, l][k % 16 / 8][row % 32][8] of the terms of
+    ``bf16_terms``, padded K), zeros past the rows and past K."""
+    rows, K = mat.shape
+    R, KP = -(-rows // 32) * 32, -(-K // 16) * 16
+    if (R, KP) != (rows, K):
+        pad = np.zeros((R, KP), np.float32)
+        pad[:rows, :K] = mat
+        mat = pad
+    img = np.empty((R // 32, KP // 16, 3, 2, 32, 8), np.uint16)
+    step = max(1, 2 ** 17 // (32 * KP))            # blocks at a time: half a megabyte stays in cache
+    for b in range(0, R // 32, step):
+        rem = mat[32 * b:32 * (b + step)].reshape(-1, 32, KP // 16, 2, 8).transpose(0, 2, 3, 1, 4)
+        bf16_terms(np.ascontiguousarray(rem, np.float32), np.moveaxis(img[b:b + step], 2, -1))
+    return img, KP
 
 
 def _check_reduce_size(M: int, N: int) -> None:
@@ -83,7 +134,7 @@ def dw_rows_per_thread(oh: int) -> int:
 class HipCodegen(Int8LoweringMixin):
     def __init__(self, schedule_fn: Optional[ScheduleFn] = None, *, conv_mode: str = "implicit",
                  int8_depthwise: str = "mfma", small_conv: bool = True,
-                 winograd="auto", pair_convs: bool = True) -> None:
+                 winograd="auto", pair_convs: bool = True, split_fp32="auto") -> None:
         """``int8_depthwise``: "mfma" runs 16-channel-aligned int8 depthwise
         convs as block-diagonal GEMMs on the matrix cores, "vector" keeps
         them on the per-pixel vector kernel. ``small_conv``: convs with few
@@ -99,7 +150,14 @@ class HipCodegen(Int8LoweringMixin):
             raise ValueError(f"conv_mode must be 'implicit' or 'im2col', not {conv_mode!r}")
         if int8_depthwise not in ("mfma", "vector"):
             raise ValueError(f"int8_depthwise must be 'mfma' or 'vector', not {int8_depthwise!r}")
+        if split_fp32 not in (True, False, "auto"):
+            raise ValueError(f"split_fp32 must be True, False or 'auto', not {split_fp32!r}")
         self.int8_depthwise_mfma = int8_depthwise == "mfma"
+        # a caller's own schedules, and winograd=False (the plain fp32 implicit
+        # GEMM), keep the fp32 instruction unless the split is asked for
+        self.split_fp32 = split_fp32 if split_fp32 != "auto" else \
+            ("auto" if schedule_fn is None and winograd is not False else False)
+        self.parts: set = set()          # library parts beyond the launch kinds'
         if schedule_fn is None:
             from mdlc_amd.autotuner.tuner import tuned_schedules
 
@@ -206,7 +264,7 @@ class HipCodegen(Int8LoweringMixin):
                 raise NotImplementedError(f"HIP codegen: no device lowering for {op!r}")
         if self.pair_convs:
             self._pair_convs(g)
-        lib = library_parts({l.kind for l in self.plan})
+        lib = library_parts({l.kind for l in self.plan}, self.parts)
         return HipModule(g, self.kernels, self.plan, self.scratch, self.consts, lib,
                          scratch_class=self.scratch_class, device_layout=dict(self.layout))
 
@@ -227,7 +285,8 @@ class HipCodegen(Int8LoweringMixin):
             return {mem.assignment[e] for e in names if e in mem.assignment}
 
         def one_slice_conv(l):
-            return (l.kind == "conv" and not l.meta.get("partial") and not l.meta.get("stream_k")
+            return (l.kind == "conv" and isinstance(l.meta["sched"], MfmaSchedule)
+                    and not l.meta.get("partial") and not l.meta.get("stream_k")
                     and l.grid[1:] == (1, 1) and l.meta.get("ksplit", 1) == 1)
 
         cus = schedule_mod.CUS
@@ -304,6 +363,10 @@ class HipCodegen(Int8LoweringMixin):
                    "batch": N, "bias": has_bias, "act": act,
                    **{k: geo[k] for k in ("C", "H", "W", "KH", "KW", "SH", "SW", "DH", "DW",
                                           "PT", "PB", "PL", "PR", "OH", "OW")}}
+        x3 = conv_x3_schedule(geo) if self.conv_mode == "implicit" and self.split_fp32 is not False else None
+        if x3 is not None and self._x3_wins(problem, x3[1]) and not self._keeps_pair(g, node, problem):
+            self._lower_conv_x3(g, node, geo, has_bias, x3[0])
+            return
         sched = self._schedule(node, (OC, P, K), problem)
         if self.conv_mode == "implicit" and sched.WK > 1 and (geo["C"] % 16 or not sched.is_valid()):
             raise ValueError(f"wave-split schedule {sched.key_full()} needs Cin % 16 == 0")
@@ -354,6 +417,104 @@ class HipCodegen(Int8LoweringMixin):
         meta.update({"ldb": ldc})
         self._emit_gemm("gemm", sched, [wdev, cols], bias, y, meta, epi, bmode=0, vec_a=True,
                         out_nchw=True)
+
+    def _x3_wins(self, problem: dict, us: float) -> bool:
+        """Whether a split-bf16 launch estimated at ``us`` replaces the fp32
+        kernel: always without a measured fp32 schedule for the problem (the
+        default schedules were slower on every shape measured, 1.1 to 2.3
+        times), else where the estimate is a fifth below its time (single-image
+        layers stay on the wave-split kernel: 3.3 against 5.0 us)."""
+        if self.split_fp32 is True:
+            return True
+        measured = getattr(self.schedule_fn, "measured_us", lambda p: None)(problem)
+        return measured is None or us < 0.8 * measured
+
+    def _keeps_pair(self, g: Graph, node: Node, problem: dict) -> bool:
+        """Whether a measured fp32 convolution can share its launch with a
+        sibling that reads the same input (``_pair_convs``; the choice of
+        kernel is the same with pairing off): ResNet's stride-2 conv and
+        downsample take 45.4 us together, 33.7 + 10.9 us apart with the first
+        on split bf16."""
+        if self.split_fp32 is True:
+            return False
+        sched = self._schedule(node, (problem["M"], problem["N"], problem["K"]), problem)
+        tiles = -(-problem["M"] // sched.BM) * -(-problem["N"] // sched.BN)
+        return (sched.SK == 1 and not sched.ST and sched.WK == 1
+                and PAIR_MIN_IDLE <= schedule_mod.CUS - tiles <= schedule_mod.CUS // 2
+                and any(n is not node and n.op_type in ("Conv", "FusedConvAct", "FusedConvBNAct")
+                        and n.inputs[0] == node.inputs[0] for n in g.nodes))
+
+    def _emit_x3(self, kind, make, sig, sched, chunk, operands, bias, out, meta, epi) -> None:
+        """Append a split-bf16 GEMM or convolution (and, with split-K, its
+        reduce launch). ``meta["K"]`` is the depth the constant is packed to,
+        ``chunk`` the depth of a slice, ``make(split, i)`` the kernel's (name,
+        source)."""
+        M, N, K = meta["M"], meta["N"], meta["K"]
+        slices = -(-K // chunk)
+        tiles = -(-M // sched.BM) * -(-N // sched.BN)
+        act, residual, res = epi["act"], epi.get("residual"), epi.get("res_input")
+        extra = [res] if res else []
+        meta = dict(meta, ksplit=slices, kchunk=chunk, ldc=epi["ldc"], hw=epi["hw"], sched=sched)
+        meta.setdefault("ldb", 0)
+        split = slices > 1
+        sig = (kind, replace(sched, SK=min(slices, 2))) + sig + \
+            (("partial",) if split else (bool(bias), epi["act_sig"], epi["alpha"], epi["beta"], residual))
+        kname = self._kernel(sig, lambda i: make(split, i))
+        block = (sched.threads_per_block(), 1, 1)
+        if not split:
+            self.plan.append(Launch(kind, kname, operands + bias + extra, [out], (tiles, 1, 1), block, meta))
+            return
+        ws = out + "__splitk"
+        self.scratch[ws] = (slices * M, N)
+        self.scratch_class[ws] = "splitk"
+        extra_bytes = 4 * (M * N * (1 + len(extra)) + (M if epi["bias_mode"] == "row" else N) * len(bias))
+        self.plan.append(Launch(kind, kname, list(operands), [ws], (tiles * slices, 1, 1), block,
+                                dict(meta, partial=True,
+                                     bytes=meta["bytes"] - extra_bytes + 4 * slices * M * N)))
+        self._emit_reduce(ws, bias, extra, out, M, N, slices, epi, meta, act,
+                          "_res" if residual else "", residual)
+
+    def _lower_conv_x3(self, g: Graph, node: Node, geo: dict, has_bias: bool, sched) -> None:
+        """A convolution on ``conv_x3``: k ordered (16-channel block, tap,
+        channel), channels padded to whole stages, the weights split and
+        packed."""
+        OC, C, KH, KW, N = geo["OC"], geo["C"], geo["KH"], geo["KW"], geo["N"]
+        OH, OW, P = geo["OH"], geo["OW"], geo["N"] * geo["OH"] * geo["OW"]
+        x, w, y, a = node.inputs[0], node.inputs[1], node.outputs[0], node.attrs
+        taps, stage = KH * KW, 16 * sched.KS
+        CP = -(-C // stage) * stage
+        wt = np.zeros((OC, CP, taps), np.float32)
+        wt[:, :C] = np.asarray(g.initializers[w], np.float32).reshape(OC, C, taps)
+        wt = wt.reshape(OC, CP // 16, 16, taps).transpose(0, 1, 3, 2).reshape(OC, CP * taps)
+        wdev, K = self._pack_x3(f"{w}__dev_x3c{stage}", wt)
+        stages = CP // stage
+        per = -(-stages // min(sched.SK, stages))
+        bias = [node.inputs[2]] if has_bias else []
+        act = a.get("activation")
+        meta = {"M": OC, "N": P, "K": K, "lda": K, "with_bias": has_bias, "node": node,
+                "weight_2d": (OC, C * taps), "out_4d": (N, OC, OH, OW), "flops": 2 * OC * P * C * taps,
+                "bytes": 4 * (N * C * geo["H"] * geo["W"] + OC * C * taps + P * OC + (OC if has_bias else 0)),
+                "Cin": C, "H": geo["H"], "W": geo["W"], "OH": OH, "OW": OW}
+        epi = dict(bias_mode="row", act=act, attrs=self._act_attrs(a), act_sig=self._act_sig(a),
+                   alpha=1.0, beta=1.0, ldc=0, hw=OH * OW, **self._residual_epilogue(g, node))
+        if epi["res_input"]:
+            meta["bytes"] += 4 * P * OC
+        win = (KH, KW, geo["SH"], geo["SW"], geo["DH"], geo["DW"], geo["PT"], geo["PL"])
+        self.parts |= {"gemm_x3", "conv_x3"}
+
+        def make(split, i):
+            tag = "SK" if split else f"{act or 'none'}{'_res' if epi['residual'] else ''}"
+            return T.conv_x3_kernel(f"conv_{sched.key()}_{tag}_{i}", replace(sched, SK=2 if split else 1), win,
+                                     with_bias=has_bias, activation=act, attrs=epi["attrs"],
+                                     residual=epi["residual"])
+
+        self._emit_x3("conv", make, (win,), sched, per * stage * taps, [wdev, x], bias, y, meta, epi)
+
+    def _pack_x3(self, name: str, mat: np.ndarray) -> tuple:
+        """A constant [rows][K] split and packed for ``gemm_x3``; returns
+        (device name, K padded to 16)."""
+        img, kp = x3_pack(mat)
+        return self._pack(name, img.view(np.float32)), kp
 
     def _lower_grouped_conv(self, g: Graph, node: Node, geo: dict, has_bias: bool) -> None:
         """A grouped convolution (1 < group, more than one input channel per
@@ -810,9 +971,19 @@ class HipCodegen(Int8LoweringMixin):
         act = a.get("activation")
         problem = {"kind": "gemm", "M": M, "N": N, "K": K, "bias": has_bias, "act": act,
                    "vec_a": vec_a, "bmode": 0 if g.is_constant(B) or N % 4 == 0 else 1}
-        sched = self._schedule(node, (M, N, K), problem)
-        b_kn = sched.WK > 1 and sched.BT and g.is_constant(B)
-        if b_kn:
+        x3 = None
+        # the kernel's operands, packed constant and output have byte offsets below 2^31 - 16
+        if (self.split_fp32 is not False and g.is_constant(B) and not g.is_constant(A)
+                and max(4 * M * K, 4 * M * N, 6 * (N + 31) * (K + 15)) < 0x7ffffff0):
+            pick, us = x3_schedule(M, N, K)
+            x3 = pick if self._x3_wins(problem, us) else None
+        sched = x3 or self._schedule(node, (M, N, K), problem)
+        b_kn = x3 is None and sched.WK > 1 and sched.BT and g.is_constant(B)
+        if x3 is not None:
+            warr = np.asarray(g.initializers[B], np.float32)
+            bdev, kp = self._pack_x3(f"{B}__dev_x3", warr if tb else warr.T)
+            ldb, bmode = 0, 0
+        elif b_kn:
             # the wave-split kernel reads constant weights K-contiguous per column
             bdev, ldb = self._pack_rows(g, B, N, K, transpose=not tb, tag="_kn")
             bmode = 0
@@ -843,6 +1014,18 @@ class HipCodegen(Int8LoweringMixin):
                 "bytes": 4 * (M * K + K * N + M * N + (N if has_bias else 0))}
         epi = dict(bias_mode="col", act=act, attrs=self._act_attrs(a), act_sig=self._act_sig(a),
                    alpha=alpha, beta=beta, ldc=N, hw=0)
+        if x3 is not None:
+            self.parts.add("gemm_x3")
+            slices, chunk = split_slices(kp, x3)
+
+            def make(split, i):
+                return T.gemm_x3_kernel(f"gemm_{x3.key()}_{'SK' if split else act or 'none'}_{i}",
+                                        replace(x3, SK=slices), with_bias=has_bias, activation=act,
+                                        attrs=epi["attrs"], alpha=alpha, beta=beta, vec=vec_a)
+
+            self._emit_x3("gemm", make, (vec_a,), x3, chunk, [adev, bdev], bias_ins, node.outputs[0],
+                          dict(meta, K=kp), epi)
+            return
         self._emit_gemm("gemm", sched, [adev, bdev], bias_ins, node.outputs[0], meta, epi,
                         bmode=bmode, vec_a=vec_a, out_nchw=False)
 
@@ -1083,6 +1266,8 @@ def wino_pack_filters(u: np.ndarray, OCP: int, CP: int) -> np.ndarray:
 
 def emit_hip_module(graph: Graph, schedule_fn: Optional[ScheduleFn] = None, *,
                     conv_mode: str = "implicit", int8_depthwise: str = "mfma",
-                    small_conv: bool = True, winograd="auto", pair_convs: bool = True) -> HipModule:
+                    small_conv: bool = True, winograd="auto", pair_convs: bool = True,
+                    split_fp32="auto") -> HipModule:
     return HipCodegen(schedule_fn, conv_mode=conv_mode, int8_depthwise=int8_depthwise,
-                      small_conv=small_conv, winograd=winograd, pair_convs=pair_convs).lower(graph)
+                      small_conv=small_conv, winograd=winograd, pair_convs=pair_convs,
+                      split_fp32=split_fp32).lower(graph)

@@ -12,7 +12,7 @@ from dataclasses import dataclass, field
 from mdlc_amd.codegen.hip import templates as T
 from mdlc_amd.ir import Graph
 
-LIBRARY_PARTS = ("common", "gemm_f32", "gemm_wsplit", "conv_wino", "conv_pool", "im2col", "pool",
+LIBRARY_PARTS = ("common", "gemm_f32", "gemm_x3", "conv_x3", "gemm_wsplit", "conv_wino", "conv_pool", "im2col", "pool",
                  "dwconv", "copy", "layout")
 QUANT_OPS = {"QuantizeLinear", "DequantizeLinear", "QConv", "QGemm", "QAdd", "QLut",
              "QGlobalAveragePool", "QMlp"}
@@ -30,10 +30,10 @@ INT8_KINDS = {"quantize", "qgemm", "qconv_first", "qmlp", "qdwconv", "qadd", "ql
               "dequantize"}
 
 
-def library_parts(kinds) -> tuple:
+def library_parts(kinds, more=()) -> tuple:
     """The library parts, in LIBRARY_PARTS order (int8 last), that launches of
-    ``kinds`` need."""
-    need = {"common", "gemm_f32"}
+    ``kinds`` need, with those of ``more``."""
+    need = {"common", "gemm_f32"} | set(more)
     for k in kinds:
         need.update(KIND_PARTS.get(k, ()))
     return tuple(p for p in LIBRARY_PARTS if p in need) + \

@@ -19,7 +19,7 @@ import os
 import re
 from typing import Optional
 
-from mdlc_amd.codegen.schedule import MfmaSchedule
+from mdlc_amd.codegen.schedule import ConvX3Schedule, MfmaSchedule, X3Schedule
 from mdlc_amd.ir import Node
 
 KERNEL_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "kernels")
@@ -198,6 +198,57 @@ def gemm_kernel(name: str, sched: MfmaSchedule, *, with_bias: bool, bias_mode: s
             f"ksplit, kchunk, {ws_val}, 0, M * hw}};\n"
             f"  {tmpl}(g);\n}}\n")
     return name, "\n".join(src)
+
+
+def gemm_x3_kernel(name: str, sched: X3Schedule, *, with_bias: bool, activation: Optional[str], attrs: dict,
+                   alpha: float = 1.0, beta: float = 1.0, vec: bool) -> tuple:
+    """(name, source) of one dense split-bf16 GEMM (``gemm_x3``): the ABI of
+    ``gemm_kernel``'s dense form with B packed, K the depth it is packed to
+    and lda A's own. ``vec``: A's depth is a multiple of 4."""
+    s = sched
+    split = s.SK > 1
+    if split:
+        with_bias, activation, alpha = False, None, 1.0
+    epi = f"{name}_epi"
+    src = epilogue_struct(epi, bias_mode="col" if with_bias else None, activation=activation,
+                          attrs=attrs, alpha=alpha, beta=beta)
+    b = {True: "true", False: "false"}
+    return name, src + (
+        f'extern "C" __global__ __launch_bounds__({s.threads_per_block()}, 2) void {name}(\n'
+        f"    const float* __restrict__ A, const float* __restrict__ B, "
+        f"{'const float* __restrict__ bias, ' if with_bias else ''}"
+        f"float* __restrict__ C,\n    int M, int N, int K, int lda, int ldb, int ldc, int hw, "
+        f"int ksplit, int kchunk) {{\n"
+        f"  mdlc::GemmArgs g{{A, B, {'bias' if with_bias else 'nullptr'}, nullptr, C, M, N, K, lda, ldb, ldc, hw, "
+        f"0, 0, 0, 0, 0, ksplit, kchunk, nullptr, 0, 0}};\n"
+        f"  mdlc::gemm_x3<{s.BM}, {s.BN}, {s.KST}, {s.WGM}, {s.WGN}, {b[s.DMA]}, {b[vec]}, "
+        f"{2 if split else 0}, {epi}>(g);\n}}\n")
+
+
+def conv_x3_kernel(name: str, sched: ConvX3Schedule, win: tuple, *, with_bias: bool,
+                   activation: Optional[str], attrs: dict, residual: Optional[str] = None) -> tuple:
+    """(name, source) of one split-bf16 convolution (``conv_x3``): the ABI of
+    ``gemm_kernel``'s conv form with the weights packed."""
+    s = sched
+    split = s.SK > 1
+    if split:
+        with_bias, residual, activation = False, None, None
+    epi = f"{name}_epi"
+    src = epilogue_struct(epi, bias_mode="row" if with_bias else None, activation=activation,
+                          attrs=attrs, residual=residual)
+    winty = "mdlc::ConvWin<%d, %d, %d, %d, %d, %d, %d, %d>" % tuple(win)
+    bias_arg = ("const float* __restrict__ bias, " if with_bias else "") + \
+        ("const float* __restrict__ res, " if residual else "")
+    bias_val = ("bias" if with_bias else "nullptr") + (", res" if residual else ", nullptr")
+    return name, src + (
+        f'extern "C" __global__ __launch_bounds__({s.threads_per_block()}) void {name}(\n'
+        f"    const float* __restrict__ A, const float* __restrict__ x, {bias_arg}"
+        f"float* __restrict__ y,\n    int M, int N, int K, int lda, int Cin, int H, int W, "
+        f"int OH, int OW, int ksplit, int kchunk) {{\n"
+        f"  mdlc::GemmArgs g{{A, x, {bias_val}, y, M, N, K, lda, 0, 0, OH * OW, Cin, H, W, OH, OW, "
+        f"ksplit, kchunk, nullptr, Cin * H * W, M * OH * OW}};\n"
+        f"  mdlc::conv_x3<{s.WGM}, {s.WGN}, {s.NI}, {s.KS}, {s.PMAX}, {s.depth(win[0] * win[1])}, "
+        f"{2 if split else 1}, {epi}, {winty}>(g);\n}}\n")
 
 
 def gemm_wsplit_kernel(name: str, sched: MfmaSchedule, *, with_bias: bool, bias_mode: str,

@@ -245,6 +245,186 @@ def default_schedule(M: int, N: int, K: int) -> MfmaSchedule:
     return s if s.conv_valid() else DEFAULT_GEMM
 
 
+# ----- the split-bf16 fp32 GEMM and convolution (gemm_x3, conv_x3) -----------------
+
+@dataclass(frozen=True)
+class X3Schedule:
+    """Tiling of ``gemm_x3``: a BM x BN tile per WGM x WGN waves of 32x32
+    blocks, KST 16-deep k steps per LDS stage, SK slices of K, B's tiles
+    through registers or (DMA) straight to LDS."""
+    BM: int = 128
+    BN: int = 128
+    KST: int = 1
+    WGM: int = 2
+    WGN: int = 2
+    SK: int = 1
+    DMA: bool = False
+
+    @property
+    def BK(self) -> int:
+        return 16 * self.KST
+
+    def threads_per_block(self) -> int:
+        return 64 * self.WGM * self.WGN
+
+    def lds_bytes(self) -> int:
+        return 2 * (self.BM + self.BN) * self.BK * 6
+
+    def valid(self) -> bool:
+        nt = self.threads_per_block()
+        return (self.BM % (32 * self.WGM) == 0 and self.BN % (32 * self.WGN) == 0
+                and self.BM * 2 * self.KST % nt == 0 and nt <= 1024 and self.lds_bytes() <= LDS_LIMIT)
+
+    def key(self) -> str:
+        return f"x3_BM{self.BM}_BN{self.BN}_K{self.BK}_W{self.WGM}x{self.WGN}{'_L' if self.DMA else ''}"
+
+
+@dataclass(frozen=True)
+class ConvX3Schedule:
+    """Tiling of ``conv_x3``: WGM x WGN waves of 32 output channels x 32 NI
+    pixels, a patch of 16 KS channels at up to PMAX positions, SK channel
+    slices."""
+    WGM: int
+    WGN: int
+    NI: int
+    KS: int
+    PMAX: int
+    SK: int = 1
+
+    @property
+    def BM(self) -> int:
+        return 32 * self.WGM
+
+    @property
+    def BN(self) -> int:
+        return 32 * self.NI * self.WGN
+
+    def threads_per_block(self) -> int:
+        return 64 * self.WGM * self.WGN
+
+    def lds_bytes(self) -> int:
+        return 2 * self.PMAX * self.KS * 96
+
+    def depth(self, taps: int) -> int:
+        """Weight k steps in registers (one less in flight): a divisor of a
+        stage's k steps."""
+        n = self.KS * taps
+        return next((d for d in (3, 4, 2, 5, 7) if n % d == 0), n)
+
+    def key(self) -> str:
+        return f"x3_BM{self.BM}_BN{self.BN}_W{self.WGM}x{self.WGN}_C{16 * self.KS}_P{self.PMAX}"
+
+
+def conv_x3_patch(geo: dict, bn: int) -> int:
+    """Positions of the largest patch over ``conv_x3``'s workgroups of ``bn``
+    pixels (the kernel's own layout: per image the rows the pixels' windows
+    touch, padded to whole strides of columns; a 1x1 convolution's are its
+    pixels)."""
+    if geo["KH"] * geo["KW"] == 1:
+        return bn
+    OH, OW, SH, SW = geo["OH"], geo["OW"], geo["SH"], geo["SW"]
+    win = (geo["KH"] - 1) * geo["DH"] + 1
+    WP = (OW - 1) * SW + (geo["KW"] - 1) * geo["DW"] + 1
+    WR = -(-WP // SW) * SW
+    FR = (OH - 1) * SH + win
+    P = geo["N"] * OH * OW
+    p0 = np.arange(0, P, bn, dtype=np.int64)
+    p1 = np.minimum(p0 + bn, P) - 1
+    nf, nl = p0 // (OH * OW), p1 // (OH * OW)
+    rlo = (p0 - nf * OH * OW) // OW * SH
+    rlast = (p1 - nl * OH * OW) // OW * SH + win
+    rows = np.where(nl == nf, rlast - rlo, FR - rlo + (nl - nf - 1) * FR + rlast)
+    return int(rows.max()) * WR
+
+
+# Estimated time of a split-bf16 launch: X3_BASE_US, plus per 16-deep k step the
+# tile's cost below times the workgroups a CU takes in turn (one workgroup
+# already keeps its CU's pipes about as busy as two), plus for a convolution
+# X3_GROUP_US for every 64-position group a wave stages, but at least the
+# operands' bytes at X3_BYTES_US; a K split adds the reduce. The costs are fits
+# over 42 GEMMs (16..4096 rows, K 384..4096) and 27 convolutions; over those the
+# pick was on average 4 % from the fastest tile measured.
+X3_BASE_US = 4.0
+X3_GROUP_US = 0.33
+X3_BYTES_US = 1 / 3.5e6                    # 3.5 TB/s, with the launch included in the base
+X3_REDUCE_US = 1.5                         # the reduce launch, plus its bytes at 8 TB/s
+X3_STEP_US = {                             # (BM, BN): us per 16-deep k step
+    (64, 64): 0.25, (64, 128): 0.48, (128, 128): 0.90, (256, 256): 2.85}
+X3_TILES = (X3Schedule(256, 256, 1, 4, 2, 1, True), X3Schedule(128, 128, 1, 2, 2),
+            X3Schedule(64, 128, 2, 2, 2), X3Schedule(64, 64, 2, 2, 2))
+CONV_X3_STEP_US = {                        # (WGM, WGN, NI)
+    (2, 2, 1): 0.21, (4, 2, 1): 0.33, (2, 4, 1): 0.33, (1, 4, 1): 0.22, (4, 2, 2): 0.66}
+CONV_X3_MAX_STEPS = 64                     # k steps a slice holds at most (1024 deep): the
+                                           # fp32 kernels split such depths, and so round less
+
+
+def x3_reduce_us(M: int, N: int, slices: int) -> float:
+    return 0.0 if slices == 1 else X3_REDUCE_US + 4 * (slices + 1) * M * N / 8e6
+
+
+def x3_schedule(M: int, N: int, K: int) -> tuple:
+    """(the dense split-bf16 schedule with the least estimated time, that
+    time in us). The 256 x 256 tile has one accumulator where the others have
+    two; it is only picked for grids that split K no less than the fp32
+    kernels do."""
+    best = None
+    for t in X3_TILES:
+        tiles = -(-M // t.BM) * -(-N // t.BN)
+        if t.BM == 256 and min(M, N) < 256:
+            continue
+        for sk in (1, 2, 3, 4, 6, 8, 12, 16):
+            s = replace(t, SK=sk)
+            slices, chunk = split_slices(-(-K // 16) * 16, s)
+            if slices != sk or (sk > 1 and (chunk < 64 or tiles * sk > 4 * CUS)):
+                continue
+            us = X3_BASE_US + -(-chunk // 16) * X3_STEP_US[t.BM, t.BN] * -(-tiles * sk // CUS) \
+                + x3_reduce_us(M, N, sk)
+            if best is None or us < best[1]:
+                best = (s, us)
+    return best
+
+
+def conv_x3_tile(geo: dict, wgm: int, wgn: int, ni: int, sk: int = 1) -> Optional[ConvX3Schedule]:
+    """The schedule of one tile for a convolution, or None where its patch
+    does not fit."""
+    ks = 1 if geo["KH"] * geo["KW"] > 1 else 2
+    pmax = -(-conv_x3_patch(geo, 32 * ni * wgn) // 64) * 64
+    s = ConvX3Schedule(wgm, wgn, ni, ks, pmax, sk)
+    groups = 2 * ks * pmax // 64
+    return s if -(-groups // (wgm * wgn)) <= 6 and s.lds_bytes() <= LDS_LIMIT else None
+
+
+def conv_x3_schedule(geo: dict) -> Optional[tuple]:
+    """(the split-bf16 convolution schedule with the least estimated time,
+    that time in us), or None where no tile fits: one group, at least eight
+    input channels, 32-bit byte offsets, fewer than 2^20 output pixels an
+    image (the kernel divides them in float)."""
+    M, N, taps = geo["OC"], geo["N"] * geo["OH"] * geo["OW"], geo["KH"] * geo["KW"]
+    inputs, outputs = geo["N"] * geo["C"] * geo["H"] * geo["W"], M * N
+    if (geo["group"] != 1 or geo["C"] < 8 or taps > 49 or geo["OH"] * geo["OW"] >= 2 ** 20
+            or 4 * max(inputs, outputs) >= 0x7ffffff0 or 6 * (M + 31) * (geo["C"] + 31) * taps >= 0x7ffffff0):
+        return None
+    best = None
+    for tile, step in CONV_X3_STEP_US.items():
+        t = conv_x3_tile(geo, *tile)
+        if t is None or (t.BM >= 2 * M and t.BM > 32):
+            continue
+        tiles = -(-M // t.BM) * -(-N // t.BN)
+        stages = -(-geo["C"] // (16 * t.KS))
+        stage_us = t.KS * taps * step + 2 * t.KS * t.PMAX / 64 / (t.WGM * t.WGN) * X3_GROUP_US
+        for sk in (1, 2, 3, 4, 6, 8, 12, 16):
+            per = -(-stages // sk)
+            if -(-stages // per) != sk or (sk > 1 and tiles * sk > 4 * CUS):
+                continue
+            if per * t.KS * taps > CONV_X3_MAX_STEPS and per > 1 and sk < 16:
+                continue
+            us = X3_BASE_US + max(per * stage_us * -(-tiles * sk // CUS),
+                                  4 * (inputs + outputs) * X3_BYTES_US) + x3_reduce_us(M, N, sk)
+            if best is None or us < best[1]:
+                best = (replace(t, SK=sk), us)
+    return best
+
+
 # ----- int8 schedules ---------------------------------------------------------
 # The same MfmaSchedule fields describe the int8 kernel, with BK counted in
 # bytes: MS = 32 selects v_mfma_i32_32x32x32_i8 (32 k per instruction), MS = 16
