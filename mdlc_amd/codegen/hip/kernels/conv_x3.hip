@@ -23,7 +23,7 @@
 // a patch from writing the next.
 //
 // Measured against the fp32 implicit GEMM: batch 8, 192 -> 320, 27x27, 3x3
-// stride 2 26.3 -> 20.8 us (error against 64 bits 3.7e-7 -> 1.4e-7); batch 32,
+// stride 2 26.3 -> 19.0 us (error against 64 bits 3.7e-7 -> 1.4e-7); batch 32,
 // 96 -> 576, 14x14, 1x1 13.2 -> 10.4 us; batch 16, 96 -> 200, 35x35, 3x3 106 ->
 // 60 us. A 128 x 128 tile keeps the matrix cores busy 64 % of its time; grids of
 // one to two workgroups a CU and the launch bound the rest.

@@ -19,25 +19,25 @@
 // float within half a bf16 ulp of FLT_MAX rounds its h to infinity. Either
 // leaves a NaN or an infinity in the accumulators, so a wave that finds one
 // there recomputes its tile with plain fp32 fmas: infinities, NaNs
-// and overflow come out as the fp32 kernel gives them. The subtractions flush
-// denormals: operands below 2^-102 lose the bits of m and l under 2^-126.
+// and overflow come out as the fp32 kernel gives them. Operands below 2^-102
+// may lose the bits of m and l under 2^-126.
 //
 // B is a constant, split and packed on the host as [32-column block][16-deep k
 // step][h, m, l][lane][8 bf16] in the instruction's lane order (lane = 32 *
 // (k % 16 / 8) + column % 32), so its tiles are copied into LDS as they are:
 // through registers two stages ahead, or (DMA) by loads straight to LDS one
 // stage ahead, where a wave's 64 x 128 tile leaves no registers. A is fp32 rows
-// of depth lda; the thread that stages eight k of a row splits them, 3.5
+// of depth lda; the thread that stages eight k of a row splits them, 5.5
 // vector instructions an element between the MFMAs, into three 16-byte LDS
 // writes. K is the depth B is packed to (zeros past A's).
 //
 // Tiling: WGM x WGN waves, each with MI x NI blocks of 32x32. LDS holds two
 // stages of KST k steps.
 //
-// Measured (fused bias + ReLU): 4096^3 1067 -> 600-650 us (256 x 256 tiles, 1.3
+// Measured (fused bias + ReLU): 4096^3 1067 -> 607 us (256 x 256 tiles, 1.36
 // PFLOP/s of bf16, what a plain bf16 product of that size reaches here; the
 // chip's power holds the clock near 1.9 GHz), error against 64 bits 1.1e-6 ->
-// 1.0e-6; 1000 x 1511 x 777 33.3 -> 26.7 us (64 x 64 tiles, two slices: vector,
+// 1.0e-6; 1000 x 1511 x 777 33.3 -> 25.4 us (64 x 64 tiles, two slices: vector,
 // LDS and matrix work of a 32-deep step take about 400 cycles each and barely
 // overlap in so small a tile), error 3.5e-7 -> 1.2e-7; 16 x 333 x 1000 17.1 ->
 // 7.3 us.
@@ -53,33 +53,26 @@ __device__ __forceinline__ unsigned cvt_bf16_pair(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
 }
 
-// A constant the compiler cannot see: folded into v_dot2 as the inline -1.0,
-// {-1, 0} was read as zero in the low half (the inline constant is a float's
-// bits, whose low half is zero).
-__device__ __forceinline__ bf16x2_t opaque_bf16x2(unsigned v) {
-  unsigned c;
-  asm("s_mov_b32 %0, %1" : "=s"(c) : "i"(v));
-  return __builtin_bit_cast(bf16x2_t, c);
-}
-
-// eight floats -> three vectors of eight bf16: h, m, l. Seven instructions a
-// pair: v_dot2_f32_bf16 with {-1, 0} and {0, -1} subtracts one half of a pair
-// exactly (11 with the halves unpacked and subtracted).
-__device__ __forceinline__ void split_bf16x3(const float (&x)[8], uintx4_t (&p)[3]) {
-  const bf16x2_t lo = opaque_bf16x2(0x0000bf80u), hi = opaque_bf16x2(0xbf800000u);
+// eight floats -> three vectors of eight bf16: h, m, l. Eleven instructions a
+// pair, all of which run beside MFMAs. (v_dot2_f32_bf16 with {-1, 0} subtracts a
+// half of a pair without unpacking it, seven instructions, but waits for the
+// matrix cores: four of them between MFMAs cost 12 ns, four additions 1 ns.
+// 4096^3 612 -> 590 us with the additions.)
+__device__ __forceinline__ void split_bf16x3_pair(float a, float b, uintx4_t (&p)[3], int j) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float a = x[2 * j], b = x[2 * j + 1];
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      const unsigned w = cvt_bf16_pair(a, b);
-      p[t][j] = w;
-      if (t < 2) {
-        a = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), lo, a, false);
-        b = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), hi, b, false);
-      }
+  for (int t = 0; t < 3; ++t) {
+    const unsigned w = cvt_bf16_pair(a, b);
+    p[t][j] = w;
+    if (t < 2) {
+      a -= __builtin_bit_cast(float, w << 16);
+      b -= __builtin_bit_cast(float, w & 0xffff0000u);
     }
   }
+}
+
+__device__ __forceinline__ void split_bf16x3(const float (&x)[8], uintx4_t (&p)[3]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) split_bf16x3_pair(x[2 * j], x[2 * j + 1], p, j);
 }
 
 // element (row, k) of a packed constant: h + m + l, the original float
