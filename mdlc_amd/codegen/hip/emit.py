@@ -49,10 +49,10 @@ from mdlc_amd.codegen.hip.emit_int8 import Int8LoweringMixin
 from mdlc_amd.codegen.hip.plan import (LIBRARY_PARTS, QUANT_OPS, HipModule, Launch,  # noqa: F401
                                        library_parts, round4, round16)
 from mdlc_amd.codegen import schedule as schedule_mod
-from mdlc_amd.codegen.schedule import (WINO_BK, WINO_BM, WINO_BN, MfmaSchedule, conv_pool_band,
+from mdlc_amd.codegen.schedule import (WINO_BK, WINO_BM, WINO_BN, WINO_X3_BK, MfmaSchedule, conv_pool_band,
                                       default_schedule, smallc_fits, smallc_pairs, smallc_tile, split_slices,
                                       unsplit_if_one_slice, wino_fits, x3_schedule, conv_x3_schedule,
-                                      wino_patch, wino_pays, wino_slices)
+                                      wino_patch, wino_pays, wino_slices, wino_x3_slices)
 from mdlc_amd.ir import DType, Graph, Node
 from mdlc_amd.passes.fuse_elementwise import ELEMENTWISE
 from mdlc_amd.passes.shape_inference import conv_geometry
@@ -342,6 +342,13 @@ class HipCodegen(Int8LoweringMixin):
                                        geo["OC"] * geo["OH"] * geo["OW"]) < 0x7ffffff0:
             self._lower_conv_smallc(g, node, geo, has_bias)
             return
+        OC, K = geo["OC"], geo["C"] * geo["KH"] * geo["KW"]
+        OH, OW, N = geo["OH"], geo["OW"], geo["N"]
+        P = N * OH * OW
+        problem = {"kind": "conv", "mode": self.conv_mode, "M": OC, "N": P, "K": K,
+                   "batch": N, "bias": has_bias, "act": act,
+                   **{k: geo[k] for k in ("C", "H", "W", "KH", "KW", "SH", "SW", "DH", "DW",
+                                          "PT", "PB", "PL", "PR", "OH", "OW")}}
         # the Winograd kernel reads its input, bias and residual through buffer
         # resources of byte offsets below 2^31 (offsets at 0x7ffffff0 read as zeros) and
         # divides tile indices and workgroup indices (at most one per channel-block,
@@ -351,18 +358,11 @@ class HipCodegen(Int8LoweringMixin):
                 and geo["N"] * geo["C"] * geo["H"] * geo["W"] * 4 < 0x7ffffff0
                 and geo["N"] * geo["OC"] * geo["OH"] * geo["OW"] * 4 < 0x7ffffff0
                 and wino_tiles < 2 ** 21
-                and -(-geo["OC"] // WINO_BM) * -(-wino_tiles // WINO_BN) * -(-geo["C"] // WINO_BK) < 2 ** 21
-                and (self.winograd is True or wino_pays(
-                    geo["OC"], geo["N"] * -(-geo["OH"] // 2) * -(-geo["OW"] // 2), geo["C"]))):
-            self._lower_wino(g, node, geo, has_bias)
-            return
-        OC, K = geo["OC"], geo["C"] * geo["KH"] * geo["KW"]
-        OH, OW, N = geo["OH"], geo["OW"], geo["N"]
-        P = N * OH * OW
-        problem = {"kind": "conv", "mode": self.conv_mode, "M": OC, "N": P, "K": K,
-                   "batch": N, "bias": has_bias, "act": act,
-                   **{k: geo[k] for k in ("C", "H", "W", "KH", "KW", "SH", "SW", "DH", "DW",
-                                          "PT", "PB", "PL", "PR", "OH", "OW")}}
+                and -(-geo["OC"] // WINO_BM) * -(-wino_tiles // WINO_BN) * -(-geo["C"] // WINO_BK) < 2 ** 21):
+            chosen = self._wino_chosen(geo, problem)
+            if self.winograd is True or chosen:
+                self._lower_wino(g, node, geo, has_bias, chosen)
+                return
         x3 = conv_x3_schedule(geo) if self.conv_mode == "implicit" and self.split_fp32 is not False else None
         if x3 is not None and self._x3_wins(problem, x3[1]) and not self._keeps_pair(g, node, problem):
             self._lower_conv_x3(g, node, geo, has_bias, x3[0])
@@ -573,7 +573,21 @@ class HipCodegen(Int8LoweringMixin):
              "bytes": 4 * (N * C * geo["H"] * geo["W"] + OC * K + P * OC * (1 + len(extra))
                            + (OC if has_bias else 0))}))
 
-    def _lower_wino(self, g: Graph, node: Node, geo: dict, has_bias: bool) -> None:
+    def _wino_chosen(self, geo: dict, problem: dict) -> bool:
+        """Whether Winograd is taken where it may be: on the grids it pays on
+        with the fp32 instruction, and where the split-bf16 convolution would
+        be taken if its own split-bf16 estimate is below that one's (measured,
+        us, Winograd against direct: 256 -> 128 channels 28x28 batch 32 56.9
+        against 104.6; 48 -> 48 56x56 batch 32 39.4 against 48.3; 144 -> 80 27x40
+        batch 9 29.0 against 26.2; 128 -> 128 28x28 batch 8 25.8 against 20.2; the
+        estimates order these and nine other shapes alike)."""
+        tiles = geo["N"] * -(-geo["OH"] // 2) * -(-geo["OW"] // 2)
+        direct = conv_x3_schedule(geo) if self.split_fp32 is not False else None
+        if direct is None or not self._x3_wins(problem, direct[1]):
+            return wino_pays(geo["OC"], tiles, geo["C"])
+        return wino_x3_slices(geo["OC"], tiles, geo["C"])[1] < direct[1]
+
+    def _lower_wino(self, g: Graph, node: Node, geo: dict, has_bias: bool, chosen: bool) -> None:
         """3x3 stride-1 conv as Winograd F(2x2, 3x3): the filters are
         transformed here (``wino_filter_transform``), the input and output
         transforms run inside the kernel. Grids too small for the chip split
@@ -583,13 +597,21 @@ class HipCodegen(Int8LoweringMixin):
         OC, OH, OW = geo["OC"], geo["OH"], geo["OW"]
         TH, TW = -(-OH // 2), -(-OW // 2)
         tiles = N * TH * TW
-        chunks = -(-C // WINO_BK)
-        nchunk = -(-chunks // wino_slices(OC, tiles, C))
+        # split bf16 where the choice was free; a grid that Winograd is forced on
+        # keeps the fp32 instruction (finer channel slices)
+        x3 = self.split_fp32 is True or (self.split_fp32 == "auto" and chosen)
+        bk = WINO_X3_BK if x3 else WINO_BK
+        chunks = -(-C // bk)
+        nchunk = -(-chunks // (wino_x3_slices(OC, tiles, C)[0] if x3 else wino_slices(OC, tiles, C)))
         slices = -(-chunks // nchunk)              # no empty slice
-        CP, OCP = slices * nchunk * WINO_BK, -(-OC // WINO_BM) * WINO_BM
+        CP, OCP = slices * nchunk * bk, -(-OC // WINO_BM) * WINO_BM
         w, x, y = node.inputs[1], node.inputs[0], node.outputs[0]
-        u = wino_pack_filters(wino_filter_transform(np.asarray(g.initializers[w])), OCP, CP)
-        udev = self._pack(f"{w}__dev_wino", u)
+        u = wino_filter_transform(np.asarray(g.initializers[w]))
+        if x3:
+            self.parts |= {"gemm_x3", "conv_wino_x3"}
+            udev = self._pack(f"{w}__dev_wino_x3", wino_x3_pack(u, OCP, CP).view(np.float32))
+        else:
+            udev = self._pack(f"{w}__dev_wino", wino_pack_filters(u, OCP, CP))
         a = node.attrs
         act = a.get("activation")
         epi = dict(act_sig=self._act_sig(a), attrs=self._act_attrs(a), **self._residual_epilogue(g, node))
@@ -610,25 +632,25 @@ class HipCodegen(Int8LoweringMixin):
         ploads = -(-wino_patch(N, H, W, geo["PT"], OH, OW) // 64)
         meta["ploads"] = ploads
         full = OH % 2 == 0 and OW % 2 == 0
-        sig = ("wino", split, ploads, full, bool(bias) and not split,
+        block = (512, 1, 1)
+        sig = ("wino", x3, split, ploads, full, bool(bias) and not split,
                None if split else epi["act_sig"], None if split else residual)
         kname = self._kernel(sig, lambda i: T.wino_kernel(
-            f"conv_wino{'_SK' if split else ''}_P{ploads}_{'none' if split else act or 'none'}{rtag}_{i}",
+            f"conv_wino{'_x3' if x3 else ''}{'_SK' if split else ''}_P{ploads}_{'none' if split else act or 'none'}{rtag}_{i}",
             split=split, ploads=ploads, full=full, with_bias=bool(bias), activation=act,
-            attrs=epi["attrs"], residual=residual))
+            attrs=epi["attrs"], residual=residual, x3=x3))
         if not split:
             if res:
                 meta["bytes"] += 4 * OC * P
             if bias:
                 meta["bytes"] += 4 * OC
-            self.plan.append(Launch("wino", kname, [udev, x] + bias + extra, [y], grid, (512, 1, 1),
-                                    meta))
+            self.plan.append(Launch("wino", kname, [udev, x] + bias + extra, [y], grid, block, meta))
             return
         ws = y + "__splitk"
         self.scratch[ws] = (slices * OC, P)
         self.scratch_class[ws] = "splitk"
         meta["bytes"] += 4 * (slices - 1) * OC * P
-        self.plan.append(Launch("wino", kname, [udev, x], [ws], grid, (512, 1, 1),
+        self.plan.append(Launch("wino", kname, [udev, x], [ws], grid, block,
                                 dict(meta, partial=True)))
         vec = REDUCE_VEC if P % 4 == 0 and (OH * OW) % 4 == 0 else 1
         _check_reduce_size(OC, P)
@@ -1262,6 +1284,28 @@ def wino_pack_filters(u: np.ndarray, OCP: int, CP: int) -> np.ndarray:
     slot_of = np.arange(2)[None, :] ^ sw[:, None]           # [lane][slot] -> quartet held
     img = img[:, :, :, :, :, lanes[:, None], slot_of, :]
     return np.ascontiguousarray(img)
+
+
+# Signs of the split-bf16 Winograd kernel's filters by position (row, column):
+# its matrix instruction rounds down on average, and with these no output sums
+# that error over all its nine positions.
+WINO_X3_SIGN = np.float32([[1], [-1], [1], [-1]]) * np.float32([1, 1, -1, 1])
+
+
+def wino_x3_pack(u: np.ndarray, OCP: int, CP: int) -> np.ndarray:
+    """U[16][OC][C] -> the split-bf16 Winograd kernel's filter operands (zero
+    padded): uint16 [OCP/64][CP/16][16 positions][2 blocks of 32][h, m, l][k %
+    16 / 8][oc % 32][8], a wave's operands of a chunk contiguous and each in
+    the lanes' order, times ``WINO_X3_SIGN`` of the position."""
+    full = np.zeros((16, OCP, CP), np.float32)
+    full[:, :u.shape[1], :u.shape[2]] = u * WINO_X3_SIGN.reshape(16, 1, 1)
+    # axes: xi, ocb, blk, li, chunk, lk, j
+    v = full.reshape(16, OCP // 64, 2, 32, CP // 16, 2, 8).transpose(1, 4, 0, 2, 5, 3, 6)
+    img = np.empty((OCP // 64, CP // 16, 16, 2, 3, 2, 32, 8), np.uint16)
+    for b in range(OCP // 64):
+        for c in range(CP // 16):
+            bf16_terms(np.ascontiguousarray(v[b, c]), np.moveaxis(img[b, c], 2, -1))
+    return img
 
 
 def emit_hip_module(graph: Graph, schedule_fn: Optional[ScheduleFn] = None, *,

@@ -12,8 +12,8 @@ from dataclasses import dataclass, field
 from mdlc_amd.codegen.hip import templates as T
 from mdlc_amd.ir import Graph
 
-LIBRARY_PARTS = ("common", "gemm_f32", "gemm_x3", "conv_x3", "gemm_wsplit", "conv_wino", "conv_pool", "im2col", "pool",
-                 "dwconv", "copy", "layout")
+LIBRARY_PARTS = ("common", "gemm_f32", "gemm_x3", "conv_x3", "gemm_wsplit", "conv_wino", "conv_wino_x3", "conv_pool",
+                 "im2col", "pool", "dwconv", "copy", "layout")
 QUANT_OPS = {"QuantizeLinear", "DequantizeLinear", "QConv", "QGemm", "QAdd", "QLut",
              "QGlobalAveragePool", "QMlp"}
 # The library parts a launch kind's kernel needs beyond "common" and

@@ -443,7 +443,8 @@ def conv_pool_kernel(name: str, win: tuple, band: int, nbx: int, *, with_bias: b
 
 
 def wino_kernel(name: str, *, split: bool, ploads: int, full: bool, with_bias: bool,
-                activation: Optional[str], attrs: dict, residual: Optional[str] = None) -> tuple:
+                activation: Optional[str], attrs: dict, residual: Optional[str] = None,
+                x3: bool = False) -> tuple:
     """3x3 stride-1 convolution by Winograd F(2x2, 3x3) on the matrix cores.
     ABI: (U, x, [bias], [res], y, int N, int C, int H, int W, int OC, int OH,
     int OW, int TH, int TW, int CP, int OCP, int PT, int PL, int nchunk) with
@@ -452,7 +453,9 @@ def wino_kernel(name: str, *, split: bool, ploads: int, full: bool, with_bias: b
     channel slices. ``split``: y is the split-K workspace and the kernel
     takes no bias or residual (``splitk_reduce_kernel`` finishes).
     ``ploads``: input patch loads per lane and channel (``wino_patch``).
-    ``full``: OH and OW are even (every 2x2 tile lies inside the output)."""
+    ``full``: OH and OW are even (every 2x2 tile lies inside the output).
+    ``x3``: the channel sums on split bf16 (``conv_wino_x3``, chunks of 16
+    channels, U packed by ``wino_x3_pack``), else in fp32 (chunks of 8)."""
     if split:
         with_bias, residual, activation = False, None, None
     epi = f"{name}_epi"
@@ -468,7 +471,7 @@ def wino_kernel(name: str, *, split: bool, ploads: int, full: bool, with_bias: b
         f"  mdlc::WinoArgs g{{U, x, {'bias' if with_bias else 'nullptr'}, "
         f"{'res' if residual else 'nullptr'}, y, N, C, H, W, OC, OH, OW, TH, TW, CP, OCP, PT, PL, "
         "nchunk};\n"
-        f"  mdlc::conv_wino_f32<{'true' if split else 'false'}, {int(ploads)}, "
+        f"  mdlc::conv_wino_{'x3' if x3 else 'f32'}<{'true' if split else 'false'}, {int(ploads)}, "
         f"{'true' if full else 'false'}, {epi}>(g);\n}}\n")
 
 

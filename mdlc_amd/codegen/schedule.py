@@ -710,6 +710,7 @@ def qconv_first_grid() -> int:
 WINO_BM = 64              # output channels per workgroup
 WINO_BN = 64              # 2x2 output tiles per workgroup
 WINO_BK = 8               # input channels per chunk
+WINO_X3_BK = 16           # and of the split-bf16 kernel
 WINO_MIN_CHUNKS = 4       # chunks each channel slice keeps at least
 
 
@@ -745,6 +746,27 @@ def wino_pays(OC: int, tiles: int, C: int) -> bool:
     blocks = -(-OC // WINO_BM) * -(-tiles // WINO_BN)
     s = wino_slices(OC, tiles, C)
     return blocks * s >= CUS // 2 and -(-C // WINO_BK) // s >= 8
+
+
+def wino_x3_slices(OC: int, tiles: int, C: int) -> tuple:
+    """(channel slices, estimated us) of the split-bf16 Winograd kernel: the
+    slice count with the least estimate, each slice keeping two chunks of 16
+    channels. A workgroup's chunk measured 2.7 us and its prologue and
+    epilogue 10 us (32 x 28x28, 64 to 192 -> 128 channels: 24.8 to 46.5 us in
+    one round of workgroups), the launch 3 us; a split adds the reduce and
+    its workspace (5 us at two slices of 6.4 MB)."""
+    blocks = -(-OC // WINO_BM) * -(-tiles // WINO_BN)
+    chunks = -(-C // WINO_X3_BK)
+    best = None
+    s = 1
+    while s == 1 or -(-chunks // s) >= 2:
+        us = 3 + -(-blocks * s // CUS) * (10 + 2.7 * -(-chunks // s))
+        if s > 1:
+            us += 4 + s * 16 * OC * tiles * X3_BYTES_US
+        if best is None or us < best[1]:
+            best = (s, us)
+        s *= 2
+    return best
 
 
 def wino_fits(geo: dict) -> bool:

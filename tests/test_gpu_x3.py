@@ -1,4 +1,5 @@
-"""The split-bf16 fp32 GEMM and convolution (``split_fp32``) on the device.
+"""The split-bf16 fp32 GEMM, convolution and Winograd convolution
+(``split_fp32``) on the device.
 
 Every tile shape at sizes that leave remainders in each dimension, against
 float64. The bound is the kernel's own: each of the six accumulations a
@@ -149,3 +150,69 @@ def test_infinities_and_nans_are_float32s(kind, hip_ctx):
     scale = np.abs(want[fin & (np.abs(want) < 1e6)]).max()
     ok = np.abs(got["y"][fin].astype(np.float64) - want[fin]) <= 1e-5 * np.maximum(np.abs(want[fin]), scale)
     assert ok.all()
+
+
+WINOS = [  # n, C, H, W, OC, pads, slices, residual
+    (3, 24, 9, 11, 40, (1, 1, 1, 1), 1, True),        # images inside a tile, odd sizes, half a chunk
+    (2, 37, 15, 13, 130, (0, 1, 2, 0), 1, False),     # ragged channels, uneven padding, three channel blocks
+    (5, 170, 7, 7, 70, (1, 1, 1, 1), 4, True),        # slices, the last one short
+    (1, 9, 30, 6, 64, (2, 2, 2, 2), 1, False),        # one chunk
+    (2, 48, 24, 56, 33, (1, 1, 1, 1), 1, True),       # even sizes: whole tiles, three chunks
+    (4, 32, 12, 64, 16, (1, 1, 1, 1), 1, False),      # the largest patches
+]
+
+
+def _wino_mag(x, w, pads):
+    """Sum over channels and positions of |U||V| (V with |B|), through |A|."""
+    U = np.abs(emit.wino_filter_transform(w)).astype(np.float64).reshape(4, 4, w.shape[0], w.shape[1])
+    x = np.pad(np.abs(x).astype(np.float64), ((0, 0), (0, 0), (pads[0], pads[2] + 1), (pads[1], pads[3] + 1)))
+    oh, ow = x.shape[2] - 3, x.shape[3] - 3
+    B = np.array([[1, 0, 1, 0], [0, 1, 1, 0], [0, 1, 1, 0], [0, 1, 0, 1]], np.float64)
+    A = np.array([[1, 1, 1, 0], [0, 1, 1, 1]], np.float64)
+    y = np.zeros((x.shape[0], w.shape[0], oh, ow))
+    for i in range(0, oh, 2):
+        for j in range(0, ow, 2):
+            d = np.pad(x[:, :, i:i + 4, j:j + 4], ((0, 0), (0, 0), (0, max(0, i + 4 - x.shape[2])),
+                                                   (0, max(0, j + 4 - x.shape[3]))))
+            v = np.einsum("ar,ncrk,bk->ncab", B, d, B)
+            m = np.einsum("aboc,ncab->noab", U, v)
+            t = np.einsum("ia,noab,jb->noij", A, m, A)
+            y[:, :, i:i + 2, j:j + 2] = t[:, :, :oh - i, :ow - j]
+    return y
+
+
+@pytest.mark.parametrize("case", WINOS, ids=lambda c: "x".join(map(str, c[:5])))
+def test_winograd(case, hip_ctx, monkeypatch):
+    """The GEMM's bound at the magnitude of Winograd's sums; U and V carry
+    three roundings more, the output transform four."""
+    n, C, H, W, OC, pads, sk, residual = case
+    monkeypatch.setattr(emit, "wino_x3_slices", lambda *a: (sk, 0.0))
+    g, feeds, w = _conv(n, C, H, W, OC, (3, 3), (1, 1), (1, 1), pads, residual)
+    cm, got, _ = device_run(g, feeds, ctx=hip_ctx, split_fp32=True, winograd=True)
+    assert "wino_x3" in cm.module.plan[0].kernel_name and (len(cm.module.plan) > 1) == (sk > 1)
+    c = g.initializers["c"].reshape(1, -1, 1, 1).astype(np.float64)
+    r = feeds.get("r", 0.0)
+    want = np.maximum(_conv64(feeds["x"], w, (1, 1), (1, 1), pads) + c + r, 0)
+    mag = _wino_mag(feeds["x"], w, pads) + np.abs(c) + np.abs(r)
+    assert np.all(np.abs(got["y"] - want) <= _bound(C + 16, mag, sk + 7))
+
+
+@pytest.mark.parametrize("sk", [1, 2])
+def test_winograd_infinities_and_nans_are_the_fp32_kernels(sk, hip_ctx, monkeypatch):
+    monkeypatch.setattr(emit, "wino_x3_slices", lambda *a: (sk, 0.0))
+    g, feeds, w = _conv(2, 70, 9, 14, 70, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, act=False)
+    x = feeds["x"]
+    x[0, 3, 0, 0], x[1, 69, 8, 13], x[1, 0, 3, 3], x[0, 40, 5, 9] = np.inf, np.nan, 3.4e38, -np.inf
+    w[67, 2, 1, 1], w[7, 50, 0, 0] = np.inf, np.nan
+    g.initializers["w"] = w
+    cm, got, _ = device_run(g, feeds, ctx=hip_ctx, split_fp32=True, winograd=True)
+    assert "wino_x3" in cm.module.plan[0].kernel_name
+    _, want, _ = device_run(g, feeds, ctx=hip_ctx, split_fp32=False, winograd=True)
+    got, want = got["y"], want["y"]
+    assert not np.isfinite(want).all() and np.isfinite(want).any()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    scale = np.abs(want[fin & (np.abs(want) < 1e6)]).max()
+    assert (np.abs(got[fin].astype(np.float64) - want[fin]) <= 1e-5 * np.maximum(np.abs(want[fin]), scale)).all()

@@ -7,9 +7,9 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from mdlc_amd.codegen.hip.emit import x3_pack
+from mdlc_amd.codegen.hip.emit import WINO_X3_SIGN, wino_x3_pack, x3_pack
 from mdlc_amd.codegen.schedule import (CONV_X3_MAX_STEPS, CONV_X3_STEP_US, conv_x3_patch, conv_x3_schedule,
-                                       conv_x3_tile, x3_schedule)
+                                       conv_x3_tile, wino_patch, wino_x3_slices, x3_schedule)
 from mdlc_amd.compiler import compile_graph
 from mdlc_amd.tools.graph_builder import GraphBuilder
 
@@ -76,6 +76,63 @@ def test_patch_covers_every_window(geo, bn):
                         n, row = nf + 1 + (q - rows0) // FR, (q - rows0) % FR
                     col = c % WPH * SW + c // WPH
                     assert (n, row, col) == (nf + s1, oh * SH + kh * geo["DH"], ow * SW + kw * geo["DW"])
+
+
+@pytest.mark.parametrize("OC,C,OCP,CP", [(5, 3, 64, 16), (70, 40, 128, 64)])
+def test_winograd_filter_image_sums_to_the_floats(OC, C, OCP, CP):
+    u = np.random.default_rng(OC).standard_normal((16, OC, C)).astype(np.float32)
+    t = (wino_x3_pack(u, OCP, CP).astype(np.uint32) << 16).view(np.float32)
+    v = t[:, :, :, :, 0] + (t[:, :, :, :, 1] + t[:, :, :, :, 2])        # ocb, chunk, xi, blk, lk, li, j
+    v = v.transpose(2, 0, 3, 5, 1, 4, 6).reshape(16, OCP, CP)
+    np.testing.assert_array_equal(v[:, :OC, :C] * WINO_X3_SIGN.reshape(16, 1, 1), u)
+    assert not v[:, OC:].any() and not v[:, :, C:].any()
+
+
+@pytest.mark.parametrize("N,H,W,PT,PL,OH,OW", [(3, 9, 11, 1, 1, 9, 11), (2, 15, 13, 0, 1, 15, 12), (5, 7, 7, 1, 1, 7, 7),
+                                               (1, 30, 5, 2, 2, 32, 7), (2, 24, 56, 1, 1, 24, 56), (40, 2, 1, 1, 0, 2, 1)])
+def test_winograd_patch_planes_hold_every_window(N, H, W, PT, PL, OH, OW):
+    """The kernel's layout: where a tile's window position is read, the pixel
+    that was loaded there."""
+    TH, TW = -(-OH // 2), -(-OW // 2)
+    TT, P, WP, SR, PW = TH * TW, N * TH * TW, 2 * TW + 2, 2 * TH + 2, TW + 1
+    size = -(-wino_patch(N, H, W, PT, OH, OW) // 64) * 64
+    for t0 in range(0, P, 64):
+        last = min(t0 + 63, P - 1)
+        nf, nl = t0 // TT, last // TT
+        rlo0, rhil = 2 * (t0 % TT // TW) - PT, 2 * (last % TT // TW) + 3 - PT
+        rows0 = (rhil if nl == nf else 2 * TH + 1 - PT) - rlo0 + 1
+        PS = rows0 * WP + ((nl - nf - 1) * SR * WP + (rhil + PT + 1) * WP if nl > nf else 0)
+        PP = PS >> 2
+        assert PS % (2 * WP) == 0 and rows0 % 2 == 0 and PS <= size
+        for t in range(t0, last + 1):
+            n, ty, tx = t // TT, t % TT // TW, t % TW
+            row = 2 * ty - PT - rlo0 if n == nf else rows0 + (n - nf - 1) * SR + 2 * ty
+            for r in range(4):
+                for k in range(4):
+                    e = (row >> 1) * PW + tx + (r & 1) * 2 * PP + (r >> 1) * PW + (k & 1) * PP + (k >> 1)
+                    pl, f = divmod(e, PP)
+                    q, col = 2 * (f // PW) + (pl >> 1), 2 * (f % PW) + (pl & 1)
+                    seg, h = (0, rlo0 + q) if q < rows0 else (1 + (q - rows0) // SR, (q - rows0) % SR - PT)
+                    assert 0 <= e < PS and (nf + seg, h, col - PL) == (n, 2 * ty - PT + r, 2 * tx - PL + k)
+
+
+def test_winograd_or_direct():
+    """Winograd where its estimate is below the direct convolution's, with
+    slices that leave two chunks each."""
+    def kernel(C, OC, H, W, batch, **kw):
+        b = GraphBuilder("g")
+        b.input("x", (batch, C, H, W))
+        b.const("w", np.ones((OC, C, 3, 3), np.float32))
+        b.node("Conv", ["x", "w"], "y", kernel_shape=[3, 3], strides=[1, 1], dilations=[1, 1], pads=[1, 1, 1, 1], group=1)
+        b.output("y")
+        return compile_graph(b.graph(), feeds={"x": np.zeros((batch, C, H, W), np.float32)}, **kw).module.plan[0].kernel_name
+
+    assert "wino_x3" in kernel(256, 128, 28, 28, 32) and "wino_x3" in kernel(128, 128, 28, 28, 32)
+    assert "conv_x3" in kernel(144, 80, 27, 40, 9) and "wino" not in kernel(128, 128, 28, 28, 8)
+    assert "wino" in kernel(144, 80, 27, 40, 9, split_fp32=False) and "x3" not in kernel(128, 128, 28, 28, 32, split_fp32=False)
+    for oc, tiles, c in [(64, 16, 16), (64, 16, 33), (512, 512, 512), (512, 16, 2048)]:
+        s, us = wino_x3_slices(oc, tiles, c)
+        assert us > 0 and (s == 1 or -(-(-(-c // 16)) // s) >= 2)
 
 
 def test_schedules_cover_k_and_fit():
