@@ -21,6 +21,8 @@ from mdlc_amd.codegen.schedule import (
 )
 from mdlc_amd.passes.shape_inference import conv_geometry
 
+QUANT_PX, QUANT_CH = 32, 64      # pixels x channels a workgroup of the layout-changing quantize turns
+
 
 def wdev_bytes(nob: int, ns: int) -> int:
     """Bytes of the first int8 conv's packed MFMA weight fragments."""
@@ -104,7 +106,10 @@ class Int8LoweringMixin:
             n, c, hw = 1, 1, int(np.prod(shp))
         self._kernel("quantize", lambda i: T.quantize_kernel("quantize_nchw_nhwc"))
         total = n * c * hw
-        self.plan.append(Launch("quantize", "quantize_nchw_nhwc", [x], [y], (-(-total // 256), 1, 1),
+        # tiles of 32 pixels x 64 channels where the order changes, else runs
+        # of four elements a thread
+        blocks = -(-total // 1024) if c == 1 or hw == 1 else n * -(-hw // QUANT_PX) * -(-c // QUANT_CH)
+        self.plan.append(Launch("quantize", "quantize_nchw_nhwc", [x], [y], (blocks, 1, 1),
                                 (256, 1, 1), {"N": n, "C": c, "HW": hw,
                                               "inv_s": float(node.attrs["inv_scale"]), "node": node,
                                               "bytes": 5 * total}))

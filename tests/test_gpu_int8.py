@@ -143,6 +143,31 @@ def test_qgemm_bit_exact(sched, out, hip_ctx):
     np.testing.assert_array_equal(got["y"], want["y"])
 
 
+@pytest.mark.parametrize("shape", [(2, 3, 5, 7), (1, 192, 14, 14), (3, 70, 9, 11), (2, 8, 4, 8), (2, 65, 3, 11),
+                                   (1, 64, 1, 1), (5, 67, 1, 1), (3, 1, 5, 7), (5, 33), (1, 4)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_quantize_bit_exact(shape, hip_ctx):
+    """Tiles with remainders of pixels and channels, whole and partial 8-channel
+    runs, and the order-keeping form; halves round to even, infinities clamp,
+    a NaN is -127."""
+    rng = np.random.default_rng(len(shape))
+    b = GraphBuilder("q")
+    b.input("x", shape)
+    b.node("QuantizeLinear", ["x"], "y", inv_scale=4.0)
+    b.output("y")
+    x = (rng.integers(-400, 400, shape) / 8).astype(np.float32)       # quotients on halves too
+    flat = x.reshape(-1)
+    flat[:3] = np.inf, -np.inf, 1e30
+    _, got, want = device_run(b.graph(), {"x": x}, ctx=hip_ctx)
+    assert got["y"].dtype == np.int8 and got["y"].shape == shape
+    np.testing.assert_array_equal(got["y"], want["y"])
+    flat[-1] = np.nan
+    with np.errstate(invalid="ignore"):
+        _, nan, _ = device_run(b.graph(), {"x": x}, ctx=hip_ctx)
+    assert nan["y"].reshape(-1)[-1] == -127
+    np.testing.assert_array_equal(nan["y"].reshape(-1)[:-1], got["y"].reshape(-1)[:-1])
+
+
 @pytest.mark.parametrize("c", [32, 192])
 def test_qadd_qlut_qgap(c, hip_ctx):
     """Add, lookup and the pool, bit-exact; C = 192 spreads each image's pool
