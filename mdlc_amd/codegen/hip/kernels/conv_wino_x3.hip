@@ -321,6 +321,9 @@ __device__ __forceinline__ void conv_wino_x3(const WinoArgs& g) {
     step(c, p0, p1);
     if (c + 1 < nch) step(c + 1, p1, p0);
   }
+  // the loads past the last chunk land in the patches, which other waves reuse
+  // after the next barrier
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- output transform, a tile half at a time -------------------------------------
   // A wave writes its positions' sums to [xi][r group][lane], four channels a
